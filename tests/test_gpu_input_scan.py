@@ -109,6 +109,38 @@ def test_scan_of_empty_boxes():
     assert (pmax.cpu() == float("-inf")).all()
 
 
+# one cell; one short of, at and past a wave's and a workgroup's run of
+# loads; the most pairs and cells of the one-launch scan and the first beyond
+# each; pairs cut into several runs
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [(1, 1, 1), (1, 1, 1023), (1, 4, 256), (1, 5, 205), (16, 63, 65), (17, 3, 5),
+                                   (64, 32, 32), (65, 32, 31), (1, 256, 256), (1, 256, 257), (3, 127, 129),
+                                   (2, 1000, 1031), (2100, 9, 7)])
+def test_scan_counts_over_sizes(shape):
+    print(f"[gpu case] ohm_scan_inputs over sizes: {shape}", flush=True)
+    x = _scores(sum(shape), shape, scale=1.0)
+    r = torch.rand(shape, generator=torch.Generator().manual_seed(3)).to(DEV)
+    x[r < 0.3] = float("-inf")
+    x[r > 0.99] = 85.0   # past the bound
+    x[(r > 0.98) & (r < 0.985)] = -1.0e4
+    x[-1, -1, -1] = float("inf")
+    x[0, 0, 0] = -3.0
+    if shape[0] > 2:
+        x[1] = float("-inf")
+    lengths = torch.full((shape[0], 2), min(shape[1:]), dtype=torch.int32, device=DEV)
+    lengths[-1, 0] = shape[1] + 1
+    # unaligned scores as well (a contiguous view one float into its storage)
+    shifted = torch.cat([x.new_zeros(1), x.reshape(-1)])[1:].view(shape)
+    for y in (x, shifted):
+        counts = torch.full((4,), 9, dtype=torch.int32, device=DEV)
+        pmax = torch.full((shape[0],), 9.0, device=DEV)
+        _lib.scan_inputs(y, lengths, 80.0, -1.0e4, counts, pmax)
+        torch.cuda.synchronize()
+        assert counts.tolist() == [int(torch.isposinf(x).sum()), int((x == 85.0).sum()),
+                                   int(torch.isneginf(x).sum()), 1]
+        assert torch.equal(pmax, x.amax(dim=(1, 2)))
+
+
 CASES = {
     "clean": lambda x: None,
     "masked_rows": lambda x: x[1, 40:, :].fill_(float("-inf")),
