@@ -1373,7 +1373,12 @@ int affine_table_stride(int ck) { return ck < kCkpt ? ck : kCkpt; }
 Geometry choose_geometry(int B, int L1max) {
     const int cus = device_cus();
     const int strips = (L1max + kStrip - 1) / kStrip;
-    int waves = (B >= 2 * cus) ? 4 : 8;
+    // 8 waves while every pair is resident at 16 waves per CU (512 pairs up to
+    // 768 x 768: 1.18 ms against 1.48 ms at 4; 2048 pairs up to 1024 x 1024:
+    // 4.43 against 3.68), and for pairs of at least 6 strips (64 pairs of 384 x
+    // 391, up to 6 strips: 0.46 ms against 0.51; 256 of 320 x 333, 5 strips: 2%
+    // slower)
+    int waves = (B <= 2 * cus && strips >= 6) ? 8 : 4;
     while (waves > 1 && waves > strips) waves >>= 1;
     int v = g_cfg_waves.load() ? g_cfg_waves.load() : env_int("OHM_WAVES", 0);
     if (v == 1 || v == 2 || v == 4 || v == 8) waves = v;
@@ -1480,6 +1485,13 @@ ohm_status setup(int op, bool affine, const float* scores, const int32_t* length
         }                                                                                 \
     } while (0)
 
+// Runs BODY with `constexpr bool SH` set to ON (shared-exponent blocks).
+#define OHM_WITH_SH(ON, BODY)                                                             \
+    do {                                                                                  \
+        if (ON) { constexpr bool SH = true; BODY; }                                       \
+        else { constexpr bool SH = false; BODY; }                                         \
+    } while (0)
+
 #define OHM_DISPATCH_W(L, KERNEL_EXPR)                                                    \
     do {                                                                                  \
         const dim3 grid_((L).geo.groups);                                                 \
@@ -1499,14 +1511,14 @@ ohm_status setup(int op, bool affine, const float* scores, const int32_t* length
 // LDS, and the reverse sweep its waves' map rings; past that size (very tall
 // pairs) the workgroup kernels run.  OHM_TEAMS=0/1 forces the choice.
 constexpr size_t kLdsLimit = 160 * 1024;
-size_t team_bwd_lds_bytes(int max_strips) {
-    return team_lds_bytes(max_strips) + (size_t)kTeamWaves * kRing * kWave * sizeof(float);
+size_t team_sweep_lds_bytes(int max_strips) {
+    return team_lds_bytes(max_strips) + (size_t)kTeamWaves * kStage * sizeof(float);
 }
 bool use_teams(int B, int max_strips) {
     const int cfg = g_cfg_teams.load();
     const int forced = cfg == 1 ? 1 : cfg == 2 ? 0 : env_int("OHM_TEAMS", -1);
     if (forced == 0) return false;
-    if (team_bwd_lds_bytes(max_strips) + sizeof(TeamLds) + 1024 > kLdsLimit) return false;
+    if (team_sweep_lds_bytes(max_strips) + sizeof(TeamLds) + 1024 > kLdsLimit) return false;
     return forced == 1 || 4 * B < device_cus();
 }
 template <typename K>
@@ -1523,13 +1535,13 @@ ohm_status launch_team(K kernel, size_t lds, const Launch& L) {
 // hand-off through global memory) for batches of few long pairs, which the
 // workgroup and team kernels would leave on a few CUs.  teams = 3 in
 // ohm_set_launch_config or OHM_GRID=0/1 force the choice.
-size_t grid_bwd_lds_bytes(int max_strips) {
-    return grid_cum_bytes(max_strips) + (size_t)kGridWaves * kRing * kWave * sizeof(float);
+size_t grid_sweep_lds_bytes(int max_strips) {
+    return grid_cum_bytes(max_strips) + (size_t)kGridWaves * kStage * sizeof(float);
 }
 // Measured on 16 pairs of 4096 x 4096: grid 6.7 ms, team kernels 21 ms.
 bool use_grid(const SwArgs& a) {
     if (!a.grid) return false;
-    if (grid_bwd_lds_bytes(a.max_strips) + sizeof(GridLds) + 1024 > kLdsLimit) return false;
+    if (grid_sweep_lds_bytes(a.max_strips) + sizeof(GridLds) + 1024 > kLdsLimit) return false;
     const int cfg = g_cfg_teams.load();
     if (cfg == 1 || cfg == 2 || cfg == 4) return false;  // an explicit other shape
     const int forced = cfg == 3 ? 1 : env_int("OHM_GRID", -1);
@@ -1580,6 +1592,13 @@ bool use_scaled(const SwArgs& a) {
     return std::fabs(a.go2) <= 120.0f && std::fabs(a.ge2) <= 120.0f;
 }
 
+// Shared-exponent blocks (see sw_affine_scaled.hiph): where a gap opened next
+// to a match and extended over a block stays inside the accepted range
+// (kShLow = 2^-64); beyond it nearly every block would be tried in vain.
+bool use_shared(const SwArgs& a) {
+    return std::fabs(a.go2) + kBlk * std::fabs(a.ge2) <= 60.0f;
+}
+
 ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths,
                         const int64_t* offsets, int B, int L1max, int L2max, float go, float ge,
                         float temp, float* value, float* map, float* g0, float* g1, float* g2,
@@ -1596,6 +1615,7 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
     L.a.g1 = g1;
     L.a.g2 = g2;
     const bool scaled = affine && use_scaled(L.a);
+    const bool shared = use_shared(L.a);
     // linear gap: exponent-tracked sweeps (per-pair workgroups), the
     // log-domain sweeps for the pairs they flag; OHM_LINEAR_SCALED=0 keeps the
     // log-domain sweeps alone
@@ -1612,22 +1632,22 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
             // one fill serves both sweeps (forward entries in words 0..2,
             // reverse entries in words 4..6 of each block)
             if ((st = launch_grid_fill(L)) != OHM_OK) return st;
-            const size_t lds = grid_cum_bytes(L.a.max_strips);
-            if (need_bwd) OHM_WITH_CK(L.ck, st = launch_grid(sw_affine_scaled_forward_grid<true, CK>, lds, L));
-            else st = launch_grid(sw_affine_scaled_forward_grid<false, kCkpt>, lds, L);
+            const size_t lds = grid_sweep_lds_bytes(L.a.max_strips);
+            if (need_bwd) OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_grid(sw_affine_scaled_forward_grid<true, CK, SH>, lds, L)));
+            else OHM_WITH_SH(shared, st = launch_grid(sw_affine_scaled_forward_grid<false, kCkpt, SH>, lds, L));
             if (st != OHM_OK) return st;
         } else if (fused) {
             Launch F = L;
             F.lds = 2 * (size_t)L.a.max_strips * sizeof(int);
-            OHM_WITH_CK(L.ck, OHM_DISPATCH_W(F, (sw_affine_scaled_fused_kernel<W, CK>)));
+            OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, OHM_DISPATCH_W(F, (sw_affine_scaled_fused_kernel<W, CK, SH>))));
         } else if (team) {
-            const size_t lds = team_lds_bytes(L.a.max_strips);
-            if (need_bwd) OHM_WITH_CK(L.ck, st = launch_team(sw_affine_scaled_forward_team<true, CK>, lds, L));
-            else st = launch_team(sw_affine_scaled_forward_team<false, kCkpt>, lds, L);
+            const size_t lds = team_sweep_lds_bytes(L.a.max_strips);
+            if (need_bwd) OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_team(sw_affine_scaled_forward_team<true, CK, SH>, lds, L)));
+            else OHM_WITH_SH(shared, st = launch_team(sw_affine_scaled_forward_team<false, kCkpt, SH>, lds, L));
             if (st != OHM_OK) return st;
         } else {
-            if (need_bwd) OHM_WITH_CK(L.ck, OHM_DISPATCH_W(L, (sw_affine_scaled_forward_kernel<true, W, CK>)));
-            else OHM_DISPATCH_W(L, (sw_affine_scaled_forward_kernel<false, W, kCkpt>));
+            if (need_bwd) OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, OHM_DISPATCH_W(L, (sw_affine_scaled_forward_kernel<true, W, CK, SH>))));
+            else OHM_WITH_SH(shared, OHM_DISPATCH_W(L, (sw_affine_scaled_forward_kernel<false, W, kCkpt, SH>)));
         }
         stage_mark(1, L.stream);
         L.a.sel = 1;
@@ -1665,15 +1685,15 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
     if (scaled) {
         L.a.sel = 0;
         if (grid) {
-            OHM_WITH_CK(L.ck, st = launch_grid(sw_affine_scaled_backward_grid<CK>,
-                                               grid_bwd_lds_bytes(L.a.max_strips), L));
+            OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_grid(sw_affine_scaled_backward_grid<CK, SH>,
+                                               grid_sweep_lds_bytes(L.a.max_strips), L)));
             if (st != OHM_OK) return st;
         } else if (team) {
-            OHM_WITH_CK(L.ck, st = launch_team(sw_affine_scaled_backward_team<CK>,
-                                               team_bwd_lds_bytes(L.a.max_strips), L));
+            OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_team(sw_affine_scaled_backward_team<CK, SH>,
+                                               team_sweep_lds_bytes(L.a.max_strips), L)));
             if (st != OHM_OK) return st;
         } else if (!fused) {
-            OHM_WITH_CK(L.ck, OHM_DISPATCH_W(L, (sw_affine_scaled_backward_kernel<W, CK>)));
+            OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, OHM_DISPATCH_W(L, (sw_affine_scaled_backward_kernel<W, CK, SH>))));
         }
         stage_mark(3, L.stream);
         L.a.sel = 1;
@@ -1683,7 +1703,7 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
     } else if (lin_scaled) {
         L.a.sel = 0;
         if (lin_grid) {
-            st = launch_grid(sw_linear_scaled_backward_grid, grid_bwd_lds_bytes(L.a.max_strips), L);
+            st = launch_grid(sw_linear_scaled_backward_grid, grid_sweep_lds_bytes(L.a.max_strips), L);
             if (st != OHM_OK) return st;
         } else {
             OHM_DISPATCH_W(L, (sw_linear_scaled_backward_kernel<W>));
@@ -2156,6 +2176,7 @@ extern "C" ohm_status ohm_embed_sw_affine_forward(const void* Q, const void* K, 
     if (!use_scaled(L.a))
         return fail(OHM_EINVAL, "gap factors outside the exponent-tracked sweeps' range "
                                 "(ohm_embed_scores, then ohm_sw_affine_forward)");
+    const bool shared = use_shared(L.a);
     L.a.value = value;
     L.a.map = map;
     L.a.g0 = grad_open;
@@ -2173,9 +2194,9 @@ extern "C" ohm_status ohm_embed_sw_affine_forward(const void* Q, const void* K, 
         hipLaunchKernelGGL(kernel, dim3(groups), dim3(64 * kW), lds, L.stream, L.a, e);
         return check_launch("embedding sweep kernel");
     };
-    if (D == 32) st = launch(embed_sw_fused_kernel<kW, 32>);
-    else if (D == 64) st = launch(embed_sw_fused_kernel<kW, 64>);
-    else st = launch(embed_sw_fused_kernel<kW, 128>);
+    if (D == 32) OHM_WITH_SH(shared, st = launch(embed_sw_fused_kernel<kW, 32, SH>));
+    else if (D == 64) OHM_WITH_SH(shared, st = launch(embed_sw_fused_kernel<kW, 64, SH>));
+    else OHM_WITH_SH(shared, st = launch(embed_sw_fused_kernel<kW, 128, SH>));
     if (st != OHM_OK) return st;
     stage_mark(1, L.stream);
     stage_mark(2, L.stream);
