@@ -195,29 +195,76 @@ def lengths_checked(lengths: Tensor, L1: int, L2: int) -> bool:
 
 def scan_applies(scores: Tensor, temp: Param, lengths: Tensor | None) -> bool:
     """Whether ``scan`` can stand in for the torch checks: a plain contiguous
-    FP32 device tensor [B, L1, L2], a Python-number temperature, int32
-    lengths on the same device, outside graph capture."""
+    FP32 device tensor [B, L1, L2], a temperature on the host or the same
+    device, int32 lengths on the same device, outside graph capture."""
     fx = torch._C._functorch
     return (isinstance(scores, Tensor) and scores.is_cuda and scores.dim() == 3
             and scores.dtype == torch.float32 and scores.is_contiguous()
             and not fx.is_batchedtensor(scores) and not fx.is_gradtrackingtensor(scores)
-            and not isinstance(temp, Tensor) and not deferred(scores)
+            and not deferred(scores) and not (isinstance(temp, Tensor) and temp.device != scores.device)
             and (lengths is None or (lengths.is_cuda and lengths.dtype == torch.int32
                                      and lengths.is_contiguous())))
 
 
+def host_params(names: tuple[str, ...], params: tuple[Param, ...], scores: Tensor) -> tuple[float, ...] | None:
+    """The scoring parameters as Python numbers, device tensors among them in
+    one read-back (checked one by one on the device, a learned gap score and
+    temperature took 60 launches and 12 read-backs: 0.6 ms of a 0.8 ms step of
+    32 pairs of 128 x 117).  None, for the torch checks and their errors, where
+    a tensor is not a plain FP32 scalar on the scores' device or a tensor
+    temperature is not finite and positive."""
+    fx = torch._C._functorch
+    tensors = [p for p in params if isinstance(p, Tensor)]
+    for p in tensors:
+        if (type(p) not in (Tensor, torch.nn.Parameter) or p.device != scores.device or p.dtype != torch.float32
+                or p.numel() != 1 or p.ndim > 1 or fx.is_batchedtensor(p) or fx.is_gradtrackingtensor(p)):
+            return None
+    if not tensors:
+        return tuple(float(p) for p in params)
+    read = iter(torch.stack([p.detach().reshape(()) for p in tensors]).tolist())
+    host = tuple(next(read) if isinstance(p, Tensor) else float(p) for p in params)
+    temp = names.index("temp")
+    if isinstance(params[temp], Tensor) and not (math.isfinite(host[temp]) and host[temp] > 0.0):
+        return None
+    return host
+
+
+def _param_values_in_domain(names: tuple[str, ...], params: tuple[Param, ...], host: tuple[float, ...],
+                            bound: float) -> None:
+    """``_param_in_domain`` of every gap on the values read back; ``bound`` is
+    DOMAIN_LIMIT temperatures rounded to FP32, as the tensor comparisons
+    round it."""
+    temp = params[names.index("temp")]
+    for name, p, v in zip(names, params, host):
+        if name == "temp":
+            continue
+        if not isinstance(p, Tensor) and not isinstance(temp, Tensor):
+            _param_in_domain(name, p, temp)
+            continue
+        if not isinstance(p, Tensor) and not math.isfinite(v):
+            raise ValueError(f"{_DOMAIN_TEXT}; {name} must be finite")
+        # (a Python number compared with a tensor rounds to FP32)
+        size = abs(v) if isinstance(p, Tensor) else float(torch.tensor(abs(v), dtype=torch.float32))
+        if not (math.isfinite(v) and size <= bound):
+            raise RuntimeError(f"{_DOMAIN_TEXT}; {name} is out of domain")
+
+
 def scan(input_name: str, scores: Tensor, names: tuple[str, ...], params: tuple[Param, ...],
-         lengths: Tensor | None, length_error: str) -> Tensor:
+         lengths: Tensor | None, length_error: str, host: tuple[float, ...] | None = None) -> Tensor:
     """``numerical_domain`` + ``mask_to_sentinel`` + the lengths range check
     for a device tensor (``scan_applies``) in one native pass over the
     scores and one read-back: the same errors in the same order (lengths,
     temperature, +inf, scores domain, parameters), and the same normalised
-    scores.  Without -inf cells the scores are returned as they are."""
+    scores.  Without -inf cells the scores are returned as they are.
+    ``host``: the parameters' values (``host_params``)."""
     from . import _lib
 
     temp = params[names.index("temp")]
-    temperature(temp)
-    t = float(temp)
+    if not isinstance(temp, Tensor):
+        temperature(temp)
+    if host is None:
+        host = tuple(float(p) for p in params)
+    t = host[names.index("temp")]
     B = scores.shape[0]
     counts = torch.empty(4, dtype=torch.int32, device=scores.device)
     pair_max = torch.empty(B, dtype=torch.float32, device=scores.device)
@@ -233,12 +280,11 @@ def scan(input_name: str, scores: Tensor, names: tuple[str, ...], params: tuple[
         raise RuntimeError(f"{input_name} contains an unsupported infinity; use -inf score masks")
     if bad:
         raise RuntimeError(f"{_DOMAIN_TEXT}; {input_name} is out of domain")
-    for name, p in zip(names, params):
-        if name != "temp":
-            _param_in_domain(name, p, temp)
+    _param_values_in_domain(names, params, host, bound)
     if not ninf:
         return scores
-    return _sentinel_from(scores, pair_max.view(B, 1, 1), t)
+    like = temperature_like(temp, scores)
+    return _sentinel_from(scores, pair_max.view(B, 1, 1), like.detach() if isinstance(like, Tensor) else like)
 
 
 __all__ = ["DOMAIN_LIMIT", "deferred", "derivative_vector", "host_scalar", "lengths_checked",

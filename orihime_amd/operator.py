@@ -41,12 +41,15 @@ _LENGTHS_RANGE = "lengths entries must lie within the padded input shape"
 
 @dataclass(frozen=True)
 class KernelCall:
-    """Inputs shared by the per-family kernel callables."""
+    """Inputs shared by the per-family kernel callables.  ``host`` holds the
+    scoring parameters as checked Python numbers where the call has read them
+    already (None: the adapter checks and reads ``params`` itself)."""
 
     primary: Tensor
     params: tuple[Param, ...]
     lengths: Tensor | None
     config: Mapping[str, Any]
+    host: tuple[float, ...] | None = None
 
 
 @dataclass(frozen=True)
@@ -105,9 +108,16 @@ def _contract_param(grad_value: Tensor, per_pair: Tensor, param: Param) -> Tenso
 # --------------------------------------------------------------------------
 
 
-def _call(op: "Operator", primary, lengths, config, params) -> KernelCall:
+_HOST = "host params"  # configuration entry that carries KernelCall.host
+
+
+def _call(op: "Operator", primary, lengths, config, params, backward: bool = False) -> KernelCall:
+    """``backward``: the parameters come back from the saved tensors, which
+    hooks may have replaced, and are read again."""
+    config = dict(config)
+    host = config.pop(_HOST, None)
     return KernelCall(primary=primary, params=tuple(params), lengths=lengths,
-                      config=MappingProxyType(dict(config)))
+                      config=MappingProxyType(config), host=None if backward else host)
 
 
 class _ValueFn(torch.autograd.Function):
@@ -193,7 +203,7 @@ class _MapFn(torch.autograd.Function):
                 ti += 1
             else:
                 params.append(p)
-        call = _call(ctx.op, _to_compute(primary.detach()), ctx.lengths, ctx.config, params)
+        call = _call(ctx.op, _to_compute(primary.detach()), ctx.lengths, ctx.config, params, backward=True)
         grad_map = _to_compute(grad_map).contiguous()
         need_params = any(
             ctx.param_is_tensor[k] and ctx.needs_input_grad[4 + k] for k in range(len(params))
@@ -271,7 +281,7 @@ class _EntropyFn(torch.autograd.Function):
                 ti += 1
             else:
                 params.append(p)
-        call = _call(ctx.op, _to_compute(primary.detach()), ctx.lengths, ctx.config, params)
+        call = _call(ctx.op, _to_compute(primary.detach()), ctx.lengths, ctx.config, params, backward=True)
         field_t = ctx.op._kernels.param_backward(call, None, "temp", None)
         g = _to_compute(grad_entropy).reshape(-1, 1, 1) * field_t
         return (None, _restore(g, primary), None, None, *([None] * len(params)))
@@ -440,15 +450,20 @@ class Operator:
         # device tensors: one native scan does the range, domain and mask
         # checks with a single read-back (the torch checks below do each
         # with reductions of their own)
+        host = None
         fast = self._length_axes in ((-2, -1), (1, 2)) and _checks.scan_applies(primary, temp, lengths)
+        if fast:
+            host = _checks.host_params(self._params, params, primary)
+            fast = host is not None
         self._validate_contract(primary, params, lengths, check_range=not fast)
         if fast:
             primary = _checks.scan(self._tensor_inputs[0], primary, self._params, params, lengths,
-                                   _LENGTHS_RANGE)
+                                   _LENGTHS_RANGE, host)
         else:
             _validate_numerical_domain(self._tensor_inputs[0], primary, self._params, params)
             primary = _normalize_masked(primary, temp)
-        return primary, params, self._config_items(config)
+        items = self._config_items(config)
+        return primary, params, items if host is None else (*items, (_HOST, host))
 
     @staticmethod
     def _needs_grad(primary: Tensor, params: tuple[Param, ...]) -> bool:

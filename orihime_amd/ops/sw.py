@@ -27,8 +27,9 @@ _PARAM_NAMES = ("gap", "temp")
 def _prepare(call: KernelCall):
     gap, temp = call.params
     warn_positive_gap(gap, "gap")
-    check_temperature(temp)
-    return (scalar(gap), scalar(temp)), resolve_lengths(call)
+    if call.host is None:
+        check_temperature(temp)
+    return call.host or (scalar(gap), scalar(temp)), resolve_lengths(call)
 
 
 def _forward_kernel(call: KernelCall) -> ForwardPass:

@@ -30,10 +30,11 @@ _PARAM_NAMES = ("gap_open", "gap_ext", "temp")
 
 def _prepare(call: KernelCall):
     go, ge, temp = call.params
-    check_temperature(temp)
+    if call.host is None:
+        check_temperature(temp)
     warn_positive_gap(go, "gap_open")
     warn_positive_gap(ge, "gap_ext")
-    return (scalar(go), scalar(ge), scalar(temp)), resolve_lengths(call)
+    return call.host or (scalar(go), scalar(ge), scalar(temp)), resolve_lengths(call)
 
 
 def _forward_pass(call: KernelCall) -> ForwardPass:

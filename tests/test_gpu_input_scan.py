@@ -219,3 +219,28 @@ def test_schema_recheck_after_in_place_lengths_change():
                                          torch.tensor(-0.5, device=DEV),
                                          torch.tensor(1.0, device=DEV), ln)
     torch.cuda.synchronize()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("go,ge,T", [(-2.0, -0.5, 1.0), (-80.0, -0.5, 1.0), (-80.00002, -0.5, 1.0), (-2.0, 9.0, 0.1),
+                                     (float("nan"), -0.5, 1.0), (-2.0, float("inf"), 1.0), (-2.0, -0.5, 0.0),
+                                     (-2.0, -0.5, float("nan")), (-2.0, -0.5, float("inf"))])
+@pytest.mark.parametrize("tensors", [(True, True, True), (True, False, False), (False, False, True)])
+def test_tensor_parameters_read_back_once_check_as_the_torch_path(monkeypatch, go, ge, T, tensors):
+    # same error or same result as the checks on the device, and no parameter
+    # is read twice
+    print(f"[gpu case] tensor params {go} {ge} {T} {tensors}", flush=True)
+    x = _scores(7, (3, 20, 24), scale=0.03)
+    x[1, 3, 4] = float("-inf")
+    params = [torch.tensor(v, device=DEV) if t else v for v, t in zip((go, ge, T), tensors)]
+    outs = []
+    for scan in (True, False):
+        if not scan:
+            monkeypatch.setattr(_checks, "scan_applies", lambda *a: False)
+        try:
+            outs.append(ohm.sw_affine(x, gap_open_score=params[0], gap_extend_score=params[1], temperature=params[2]))
+        except (RuntimeError, ValueError) as exc:
+            outs.append(f"{type(exc).__name__}: {exc}")
+    torch.cuda.synchronize()
+    a, b = outs
+    assert (a == b) if isinstance(b, str) else torch.equal(a, b)
