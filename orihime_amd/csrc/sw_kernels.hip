@@ -655,10 +655,14 @@ struct SwArgs {
 // Claim the next pair for this workgroup (largest first).  Returns -1 when done.
 // All threads must call it.  The leading barrier orders the claim after every
 // wave's use of the previous one (s_pair, the progress counters).
-template <int W>
-DEV int claim_pair(const SwArgs& a, int* s_pair, int* prog, int slot) {
+struct NoHand {
+    __device__ __forceinline__ void reset(int) {}
+};
+template <int W, typename Hand = NoHand>
+DEV int claim_pair(const SwArgs& a, int* s_pair, int* prog, int slot, Hand* hand = nullptr) {
     __syncthreads();
     if (tid_x() == 0) *s_pair = atomicAdd(&a.claims[slot], 1);
+    if (hand) hand->reset(tid_x());
     for (int q = tid_x(); q < a.max_strips; q += 64 * W) prog[q] = 0;
     __syncthreads();
     // wave-uniform from here on: descriptor loads and buffer resources derived
@@ -1073,6 +1077,7 @@ __global__ __launch_bounds__(W * 64) void sw_affine_backward_kernel(SwArgs a) {
 #include "sv_affine.hiph"
 #include "sv_tangent.hiph"
 #include "sw_teams.hiph"
+#include "sw_hand.hiph"
 #include "sw_grid.hiph"
 #include "sw_affine_scaled.hiph"
 #include "sw_linear_scaled.hiph"
@@ -1541,7 +1546,7 @@ size_t grid_sweep_lds_bytes(int max_strips) {
 // Measured on 16 pairs of 4096 x 4096: grid 6.7 ms, team kernels 21 ms.
 bool use_grid(const SwArgs& a) {
     if (!a.grid) return false;
-    if (grid_sweep_lds_bytes(a.max_strips) + sizeof(GridLds) + 1024 > kLdsLimit) return false;
+    if (grid_sweep_lds_bytes(a.max_strips) + sizeof(GridLds) + sizeof(GroupHand) + 1024 > kLdsLimit) return false;
     const int cfg = g_cfg_teams.load();
     if (cfg == 1 || cfg == 2 || cfg == 4) return false;  // an explicit other shape
     const int forced = cfg == 3 ? 1 : env_int("OHM_GRID", -1);
@@ -1563,6 +1568,18 @@ ohm_status launch_grid(K kernel, size_t lds, const Launch& L) {
     const long want = ((long)L.a.B * L.a.max_strips + kGridWaves - 1) / kGridWaves;
     const long groups = std::max(1L, std::min(want, (long)device_cus() * (16 / kGridWaves)));
     hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(64 * kGridWaves), lds, L.stream, L.a);
+    return check_launch("grid kernel");
+}
+// The same for the kernels of grid_run_groups: one workgroup per four strips.
+template <typename K>
+ohm_status launch_groups(K kernel, size_t lds, const Launch& L) {
+    if (lds > 64 * 1024 &&
+        hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+        return fail(OHM_ELAUNCH, "cannot reserve LDS for the grid kernel");
+    const long want = (long)L.a.B * ((L.a.max_strips + kGroupStrips - 1) / kGroupStrips);
+    const long groups = std::max(1L, std::min(want, 4L * device_cus()));
+    hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(kGroupThreads), lds, L.stream, L.a);
     return check_launch("grid kernel");
 }
 
@@ -1633,8 +1650,8 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
             // reverse entries in words 4..6 of each block)
             if ((st = launch_grid_fill(L)) != OHM_OK) return st;
             const size_t lds = grid_sweep_lds_bytes(L.a.max_strips);
-            if (need_bwd) OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_grid(sw_affine_scaled_forward_grid<true, CK, SH>, lds, L)));
-            else OHM_WITH_SH(shared, st = launch_grid(sw_affine_scaled_forward_grid<false, kCkpt, SH>, lds, L));
+            if (need_bwd) OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_groups(sw_affine_scaled_forward_grid<true, CK, SH>, lds, L)));
+            else OHM_WITH_SH(shared, st = launch_groups(sw_affine_scaled_forward_grid<false, kCkpt, SH>, lds, L));
             if (st != OHM_OK) return st;
         } else if (fused) {
             Launch F = L;
@@ -1685,7 +1702,7 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
     if (scaled) {
         L.a.sel = 0;
         if (grid) {
-            OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_grid(sw_affine_scaled_backward_grid<CK, SH>,
+            OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_groups(sw_affine_scaled_backward_grid<CK, SH>,
                                                grid_sweep_lds_bytes(L.a.max_strips), L)));
             if (st != OHM_OK) return st;
         } else if (team) {
