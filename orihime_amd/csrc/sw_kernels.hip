@@ -1080,7 +1080,6 @@ __global__ __launch_bounds__(W * 64) void sw_affine_backward_kernel(SwArgs a) {
 #include "sw_hand.hiph"
 #include "sw_grid.hiph"
 #include "sw_affine_scaled.hiph"
-#include "sw_linear_scaled.hiph"
 #include "embed_fused.hiph"
 
 // ==========================================================================
@@ -1380,11 +1379,13 @@ Geometry choose_geometry(int B, int L1max) {
     const int strips = (L1max + kStrip - 1) / kStrip;
     // 8 waves while every pair is resident at 16 waves per CU (512 pairs up to
     // 768 x 768: 1.18 ms against 1.48 ms at 4; 2048 pairs up to 1024 x 1024:
-    // 4.43 against 3.68), and for pairs of at least 6 strips (64 pairs of 384 x
-    // 391, up to 6 strips: 0.46 ms against 0.51; 256 of 320 x 333, 5 strips: 2%
-    // slower)
-    int waves = (B <= 2 * cus && strips >= 6) ? 8 : 4;
-    while (waves > 1 && waves > strips) waves >>= 1;
+    // 4.43 against 3.68), from 5 strips (256 pairs of 320 x 333: 744 us against
+    // 753) or, past one pair per CU, 6; there rounded up to the strips, a pair's
+    // strips then run at once (256 pairs up to 384 x 400, 6 strips: 603 us at 8
+    // waves, 644 at 4)
+    const bool resident = B <= 2 * cus;
+    int waves = (resident && strips >= (B <= cus ? 5 : 6)) ? 8 : 4;
+    while (waves > 1 && (resident ? waves / 2 : waves - 1) >= strips) waves >>= 1;
     int v = g_cfg_waves.load() ? g_cfg_waves.load() : env_int("OHM_WAVES", 0);
     if (v == 1 || v == 2 || v == 4 || v == 8) waves = v;
     int per_cu = 16 / waves;
@@ -1509,12 +1510,12 @@ ohm_status setup(int op, bool affine, const float* scores, const int32_t* length
     } while (0)
 
 // Team kernels (wave-level strip scheduling, one workgroup of kTeamWaves
-// waves per CU) pay off for batches of few large pairs (measured: 4096-long
-// pairs, 16 per batch, 10% faster); for batches with at least a quarter as
-// many pairs as CUs the per-pair workgroup kernels are faster (256 x 512^2
-// and ragged batches: 15-20%).  They hold per-slot progress counters and partials in
-// LDS, and the reverse sweep its waves' map rings; past that size (very tall
-// pairs) the workgroup kernels run.  OHM_TEAMS=0/1 forces the choice.
+// waves per CU) run where OHM_TEAMS=1 or ohm_set_launch_config asks for them:
+// few long pairs are faster on the grid kernels, few short ones in one fused
+// launch (8 of 64 x 64: 106 us against 122), larger batches in per-pair
+// workgroups (256 x 512^2 and ragged batches: 15-20%).  They hold per-slot
+// progress counters and partials in LDS, and the reverse sweep its waves' map
+// rings; past that size (very tall pairs) the workgroup kernels run.
 constexpr size_t kLdsLimit = 160 * 1024;
 size_t team_sweep_lds_bytes(int max_strips) {
     return team_lds_bytes(max_strips) + (size_t)kTeamWaves * kStage * sizeof(float);
@@ -1524,7 +1525,7 @@ bool use_teams(int B, int max_strips) {
     const int forced = cfg == 1 ? 1 : cfg == 2 ? 0 : env_int("OHM_TEAMS", -1);
     if (forced == 0) return false;
     if (team_sweep_lds_bytes(max_strips) + sizeof(TeamLds) + 1024 > kLdsLimit) return false;
-    return forced == 1 || 4 * B < device_cus();
+    return forced == 1;
 }
 template <typename K>
 ohm_status launch_team(K kernel, size_t lds, const Launch& L) {
@@ -1616,6 +1617,49 @@ bool use_shared(const SwArgs& a) {
     return std::fabs(a.go2) + kBlk * std::fabs(a.ge2) <= 60.0f;
 }
 
+// The fused sweeps with checkpoints fetched a block ahead (up to 256
+// registers): where the launch has at most 8 waves per CU anyway.  Steps,
+// with and without: 256 pairs of 512 x 512 769 and 831 us, global 256 pairs up
+// to 384 x 400 610 and 725, Saigo-Vert 256 of 320 x 333 753 and 822, map of 8
+// of 64 x 64 106 and 109.  (At 16 waves per CU the same prefetch spills: 2048
+// ragged pairs 5.3 ms instead of 3.8.)
+bool use_ahead(const Launch& L) {
+    const int cus = device_cus(), groups = L.geo.groups;
+    return (groups + cus - 1) / cus * L.geo.waves <= 8;
+}
+// Whether a call of the linear, Saigo-Vert or global model runs the
+// exponent-tracked sweeps (the log-domain ones redo the pairs they flag).
+// The Saigo-Vert and global models have them in shared-exponent form only.
+bool use_model(const SwArgs& a, int model) {
+    if (!use_scaled(a)) return false;
+    if (model == kSwLinear && env_int("OHM_LINEAR_SCALED", 1) == 0) return false;
+    if (model != kSwLinear && !use_shared(a)) return false;
+    // (the fused launch's progress words)
+    return 2 * (size_t)a.max_strips * sizeof(int) <= 48 * 1024;
+}
+template <int MODEL, bool SH>
+ohm_status launch_model(const Launch& L, bool need_bwd) {
+    ohm_status st = OHM_OK;
+    if (use_grid(L.a)) {
+        // one fill serves both sweeps (forward entries in words 0..2, reverse
+        // entries in words 4..6 of each block)
+        if ((st = launch_grid_fill(L)) != OHM_OK) return st;
+        const size_t lds = grid_sweep_lds_bytes(L.a.max_strips);
+        if (!need_bwd) return launch_groups(scaled_forward_grid<MODEL, false, SH>, lds, L);
+        if ((st = launch_groups(scaled_forward_grid<MODEL, true, SH>, lds, L)) != OHM_OK) return st;
+        return launch_groups(scaled_backward_grid<MODEL, SH>, lds, L);
+    }
+    if (need_bwd) {
+        Launch F = L;
+        F.lds = 2 * (size_t)L.a.max_strips * sizeof(int);
+        if (SH && use_ahead(F)) OHM_DISPATCH_W(F, (sw_affine_scaled_fused_ahead_kernel<MODEL, W>));
+        else OHM_DISPATCH_W(F, (scaled_fused_kernel<MODEL, W, SH>));
+    } else {
+        OHM_DISPATCH_W(L, (scaled_value_kernel<MODEL, W, SH>));
+    }
+    return check_launch("scaled sweeps");
+}
+
 ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths,
                         const int64_t* offsets, int B, int L1max, int L2max, float go, float ge,
                         float temp, float* value, float* map, float* g0, float* g1, float* g2,
@@ -1633,11 +1677,10 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
     L.a.g2 = g2;
     const bool scaled = affine && use_scaled(L.a);
     const bool shared = use_shared(L.a);
-    // linear gap: exponent-tracked sweeps (per-pair workgroups), the
-    // log-domain sweeps for the pairs they flag; OHM_LINEAR_SCALED=0 keeps the
-    // log-domain sweeps alone
-    const bool lin_scaled = !affine && use_scaled(L.a) && env_int("OHM_LINEAR_SCALED", 1) != 0;
-    const bool lin_grid = lin_scaled && use_grid(L.a);
+    // linear gap: exponent-tracked sweeps, the log-domain sweeps for the pairs
+    // they flag; OHM_LINEAR_SCALED=0 keeps the log-domain sweeps alone
+    const bool shared_linear = 9.0f * std::fabs(L.a.go2) <= 60.0f;  // as use_shared: a gap's every step opens
+    const bool lin_scaled = !affine && use_model(L.a, kSwLinear);
     const bool grid = scaled && use_grid(L.a);
     const bool fused = scaled && !grid && need_bwd && use_fused(B, L.a.max_strips);
     const bool team = scaled && !grid && !fused && use_teams(B, L.a.max_strips);
@@ -1656,7 +1699,8 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
         } else if (fused) {
             Launch F = L;
             F.lds = 2 * (size_t)L.a.max_strips * sizeof(int);
-            OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, OHM_DISPATCH_W(F, (sw_affine_scaled_fused_kernel<W, CK, SH>))));
+            if (shared && L.ck == kCkpt && use_ahead(F)) OHM_DISPATCH_W(F, (sw_affine_scaled_fused_ahead_kernel<kSwAffine, W>));
+            else OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, OHM_DISPATCH_W(F, (sw_affine_scaled_fused_kernel<W, CK, SH>))));
         } else if (team) {
             const size_t lds = team_sweep_lds_bytes(L.a.max_strips);
             if (need_bwd) OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_team(sw_affine_scaled_forward_team<true, CK, SH>, lds, L)));
@@ -1674,19 +1718,8 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
         if (need_bwd) OHM_DISPATCH_W(L, (sw_affine_forward_kernel<true, W>));
         else OHM_DISPATCH_W(L, (sw_affine_forward_kernel<false, W>));
     } else if (lin_scaled) {
-        if (lin_grid) {
-            // one fill serves both sweeps (forward entries in words 0..1,
-            // reverse entries in words 4..6 of each block)
-            if ((st = launch_grid_fill(L)) != OHM_OK) return st;
-            const size_t lds = grid_cum_bytes(L.a.max_strips);
-            if (need_bwd) st = launch_grid(sw_linear_scaled_forward_grid<true>, lds, L);
-            else st = launch_grid(sw_linear_scaled_forward_grid<false>, lds, L);
-            if (st != OHM_OK) return st;
-        } else if (need_bwd) {
-            OHM_DISPATCH_W(L, (sw_linear_scaled_forward_kernel<true, W>));
-        } else {
-            OHM_DISPATCH_W(L, (sw_linear_scaled_forward_kernel<false, W>));
-        }
+        OHM_WITH_SH(shared_linear, st = (launch_model<kSwLinear, SH>(L, need_bwd)));
+        if (st != OHM_OK) return st;
         stage_mark(1, L.stream);
         L.a.sel = 1;
         if (need_bwd) OHM_DISPATCH_W(L, (sw_forward_kernel<true, W>));
@@ -1718,13 +1751,6 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
     } else if (affine) {
         OHM_DISPATCH_W(L, (sw_affine_backward_kernel<W>));
     } else if (lin_scaled) {
-        L.a.sel = 0;
-        if (lin_grid) {
-            st = launch_grid(sw_linear_scaled_backward_grid, grid_sweep_lds_bytes(L.a.max_strips), L);
-            if (st != OHM_OK) return st;
-        } else {
-            OHM_DISPATCH_W(L, (sw_linear_scaled_backward_kernel<W>));
-        }
         stage_mark(3, L.stream);
         L.a.sel = 1;
         OHM_DISPATCH_W(L, (sw_backward_kernel<W>));
@@ -1756,6 +1782,10 @@ ohm_status nw_forward_impl(const float* scores, const int32_t* lengths, const in
     L.a.g1 = g1;
     L.a.g2 = g2;
     L.a.gap_sum = gap_sum ? 1 : 0;
+    if (use_model(L.a, kNwAffine)) {
+        if ((st = launch_model<kNwAffine, true>(L, need_bwd)) != OHM_OK) return st;
+        L.a.sel = 1;
+    }
     if (need_bwd) OHM_DISPATCH_W(L, (nw_affine_forward_kernel<true, W>));
     else OHM_DISPATCH_W(L, (nw_affine_forward_kernel<false, W>));
     stage_mark(1, L.stream);
@@ -1851,6 +1881,10 @@ ohm_status sv_forward_impl(const float* scores, const int32_t* lengths, const in
     L.a.g1 = g1;
     L.a.g2 = g2;
     L.a.gap_sum = gap_sum ? 1 : 0;
+    if (use_model(L.a, kSvAffine)) {
+        if ((st = launch_model<kSvAffine, true>(L, need_bwd)) != OHM_OK) return st;
+        L.a.sel = 1;
+    }
     if (need_bwd) OHM_DISPATCH_W(L, (sv_affine_forward_kernel<true, W>));
     else OHM_DISPATCH_W(L, (sv_affine_forward_kernel<false, W>));
     stage_mark(1, L.stream);
