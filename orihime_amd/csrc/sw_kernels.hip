@@ -1382,9 +1382,14 @@ Geometry choose_geometry(int B, int L1max) {
     // 4.43 against 3.68), from 5 strips (256 pairs of 320 x 333: 744 us against
     // 753) or, past one pair per CU, 6; there rounded up to the strips, a pair's
     // strips then run at once (256 pairs up to 384 x 400, 6 strips: 603 us at 8
-    // waves, 644 at 4)
+    // waves, 644 at 4).  2 waves past the 4 pairs a CU that 4 waves each hold
+    // resident, up to 4 strips (a last round of few pairs costs the most there:
+    // 1280 pairs of 250 x 250 287 us against 334 for the value, 745 against 925
+    // for the map; 2048 of 256 x 256 912 against 1073; 1024 of 256 x 243 231
+    // against 217, 1536 of 400 x 400 693 against 627)
     const bool resident = B <= 2 * cus;
     int waves = (resident && strips >= (B <= cus ? 5 : 6)) ? 8 : 4;
+    if (B > 4 * cus && strips <= 4) waves = 2;
     while (waves > 1 && (resident ? waves / 2 : waves - 1) >= strips) waves >>= 1;
     int v = g_cfg_waves.load() ? g_cfg_waves.load() : env_int("OHM_WAVES", 0);
     if (v == 1 || v == 2 || v == 4 || v == 8) waves = v;
