@@ -744,32 +744,14 @@ def _tune(torch, launch, params, args):
             "tuning_s": round(time.perf_counter() - t0, 2)}
 
 
-def nw_traffic(kernel: str, family: str = "nw"):
-    """HBM bytes per launch of the NW (SV) forward or reverse sweep from the
-    committed FETCH_SIZE / WRITE_SIZE profile of the workload, or None."""
-    path = os.path.join(ROOT, "profiles", f"{family}_affine_ragged2048_hbm_traffic.md")
-    if not os.path.exists(path):
-        return None
-    for line in open(path):
-        if line.startswith("traffic_bytes_per_launch:"):
-            table = json.loads(line.split(":", 1)[1])
-            key = (f"{family}_affine_forward_kernel<true" if kernel == "forward"
-                   else f"{family}_affine_backward_kernel")
-            for k, v in table.items():
-                if k.startswith(key):
-                    return int(v)
-    return None
-
-
 def nw_workload(torch, args, dev, hip, family="nw"):
     """Needleman-Wunsch (family "nw") or Saigo-Vert ("sv") affine fwd+bwd on
     the ragged batch of the headline workload (2048 pairs, L1, L2 ~ U[64,
-    1024], seed 2, go=-8 ge=-0.5 T=0.5, packed layout).  Roofline: the forward
-    streams the scores in and the table out (NW: two planes, M - I and D - I;
-    SV: three, M, I - M, D - M), the reverse streams the table and the scores
-    in and the map out: 12 / 16 B per cell (NW), 16 / 20 (SV)."""
+    1024], seed 2, go=-8 ge=-0.5 T=0.5, packed layout).  Roofline: one fused
+    launch reads the scores and writes the map, 8 B per cell; the "reverse"
+    interval holds the log-domain launches, which return at once when no pair
+    was flagged."""
     from orihime_amd import _lib, ragged
-    planes = 2 if family == "nw" else 3
     call = _lib.nw_affine_forward if family == "nw" else _lib.sv_affine_forward
     ws_fn = _lib._ws_nw_affine if family == "nw" else _lib._ws_sv_affine
     params = (-8.0, -0.5, 0.5)
@@ -797,13 +779,10 @@ def nw_workload(torch, args, dev, hip, family="nw"):
     kd = kernel_durations(torch, _lib, hip, launch, max(3, min(args.steps, 10)))
     fwd_ms, rev_ms = kd["forward"], kd["reverse"]
     gcups = cells / (ms * 1e-3) / 1e9
-    byts = {"forward": (4.0 + 4 * planes) * cells, "reverse": (8.0 + 4 * planes) * cells}
-    dom = "reverse" if rev_ms >= fwd_ms else "forward"
-    dom_ms = rev_ms if dom == "reverse" else fwd_ms
-    achieved = byts[dom] / (dom_ms * 1e-3) / 1e9
-    log(f"{family} affine fwd+bwd: {ms:.3f} ms/step, {gcups:.1f} GCUPS; forward {fwd_ms:.3f} ms "
-        f"({byts['forward'] / fwd_ms / 1e6:.0f} GB/s), reverse {rev_ms:.3f} ms "
-        f"({byts['reverse'] / rev_ms / 1e6:.0f} GB/s)")
+    byts = 8.0 * cells
+    achieved = byts / (fwd_ms * 1e-3) / 1e9
+    log(f"{family} affine fwd+bwd: {ms:.3f} ms/step, {gcups:.1f} GCUPS; sweeps {fwd_ms:.3f} ms "
+        f"({achieved:.0f} GB/s algorithmic), log-domain launches {rev_ms:.3f} ms")
     line = {
         "metric": f"GCUPS soft-{family.upper()}-affine fwd+bwd (value, map, parameter grads), 1 GPU",
         "value": round(gcups, 3), "unit": "GCUPS", "n_gpus": 1, "steps": args.steps,
@@ -813,10 +792,10 @@ def nw_workload(torch, args, dev, hip, family="nw"):
                                "U[64,1024] (seed 2), gap_open=-8 gap_extend=-0.5 T=0.5, packed",
                    "cells": cells, "wall_ms_per_step": round(wall, 4),
                    "kernel_ms": {k: round(v, 4) for k, v in kd.items()}},
-        "roofline": {"bound": "hbm", "kernel": f"{family}_affine_{dom}",
+        "roofline": {"bound": "hbm", "kernel": "scaled_fused_kernel",
                      "achieved": round(achieved, 1), "peak": 8000.0, "unit": "GB/s",
-                     "frac": round(achieved / 8000.0, 4), "traffic": nw_traffic(dom, family),
-                     "bytes_per_cell": int(byts[dom] / cells)},
+                     "frac": round(achieved / 8000.0, 4), "traffic": None,
+                     "bytes_per_cell": 8},
         "cpu_baseline": None,
     }
     # the HVP along an N(0,1) direction (forward-over-reverse pass) on the same batch
