@@ -1,0 +1,125 @@
+"""Excluded cells next to strong matches: a block of steps that the forward
+sweep accepts with one exponent per lane may have to be redone by the reverse
+sweep (its adjoints climb faster than the cells), starting from cells that are
+exactly zero.  Every model and launch shape, value, map and parameter
+gradients, against the FP64 oracle at the tolerances of the parity tests."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import orihime_amd as ohm
+from helpers import abs_err, rel_err
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+ORACLE = {"sw": O.sw_forward, "sw_affine": O.sw_affine_forward, "sv_affine": O.sv_affine_forward,
+          "nw_affine": O.nw_affine_forward}
+T = 1.0
+
+
+def _hole(B, L1, L2):
+    """Weak background, strong matches one below the diagonal, one cell excluded."""
+    s = np.full((B, L1, L2), -3.0, np.float32)
+    n = min(L1 - 1, L2)
+    s[:, np.arange(n) + 1, np.arange(n)] = 5.0
+    mask = np.zeros(s.shape, bool)
+    mask[:, 0, 0] = True
+    return s, mask
+
+
+def _strong(B, L1, L2, match, seed):
+    rng = np.random.default_rng([seed, B, L1, L2])
+    s = (rng.normal(size=(B, L1, L2)) * 1.5 - 1.0).astype(np.float32)
+    n = min(L1, L2)
+    s[:, np.arange(n), np.arange(n)] += np.float32(match)
+    return s, np.zeros(s.shape, bool), rng
+
+
+def _columns(B, L1, L2, width, match=7.0):
+    s, mask, _ = _strong(B, L1, L2, match, width)
+    mask[:, :, :width] = True
+    return s, mask
+
+
+def _rows(B, L1, L2, width, match=7.0):
+    s, mask, _ = _strong(B, L1, L2, match, width)
+    mask[:, :width] = True
+    return s, mask
+
+
+def _scattered(B, L1, L2, match):
+    s, mask, rng = _strong(B, L1, L2, match, 3)
+    return s, rng.random(s.shape) < 0.2
+
+
+def _noise(B, L1, L2, scale):
+    rng = np.random.default_rng([4, B, L1, L2])
+    s = np.clip(rng.normal(size=(B, L1, L2)) * scale, -75, 75).astype(np.float32)
+    return s, rng.random(s.shape) < 0.1
+
+
+def _inside(B, L1, L2, match=7.0):
+    """A hole across the matches and the last corner left out (global: paths
+    past it are trailing gaps)."""
+    s, mask, _ = _strong(B, L1, L2, match, 5)
+    mask[:, 10:19, 5:30] = True
+    mask[:, (3 * L1) // 4:, (3 * L2) // 4:] = True
+    return s, mask
+
+
+CASES = {
+    "hole": lambda: _hole(2, 64, 64),
+    "column1": lambda: _columns(2, 70, 90, 1),
+    "columns5": lambda: _columns(2, 150, 141, 5),
+    "columns8": lambda: _columns(2, 64, 100, 8, 8.0),
+    "columns70": lambda: _columns(2, 270, 200, 70),
+    "rows1": lambda: _rows(2, 90, 70, 1),
+    "rows8": lambda: _rows(2, 150, 141, 8, 8.0),
+    "rows70": lambda: _rows(2, 200, 270, 70),
+    "scattered": lambda: _scattered(24, 130, 120, 7.0),
+    "noise8": lambda: _noise(8, 100, 90, 8.0),
+    "noise15": lambda: _noise(8, 100, 90, 15.0),
+    "inside": lambda: _inside(2, 150, 160),
+}
+# the launch shapes: one launch per pair, groups of strips and, of the affine
+# model, separate launches and teams
+SHAPES = {"fused": {"OHM_GRID": "0"}, "grid": {"OHM_GRID": "1"}, "separate": {"OHM_GRID": "0", "OHM_FUSED": "0"},
+          "team": {"OHM_GRID": "0", "OHM_FUSED": "0", "OHM_TEAMS": "1"}}
+
+
+@pytest.mark.parametrize("kind", list(CASES))
+@pytest.mark.parametrize("family,shape", [(f, x) for f in ORACLE for x in SHAPES
+                                          if f == "sw_affine" or x in ("fused", "grid")])
+def test_excluded_cells_match_the_oracle(family, kind, shape, monkeypatch):
+    print("excluded cells", family, kind, shape, flush=True)
+    for k, v in SHAPES[shape].items():
+        monkeypatch.setenv(k, v)
+    s, mask = CASES[kind]()
+    go, ge = (-1.0, 0.0) if family == "sw" else (-11.0, -1.0)
+    x = torch.from_numpy(s).cuda().requires_grad_()
+    p = [torch.tensor(v, device="cuda", requires_grad=True) for v in ((go, T) if family == "sw" else (go, ge, T))]
+    kw = dict(zip(("gap_score", "temperature") if family == "sw" else
+                  ("gap_open_score", "gap_extend_score", "temperature"), p), mask=torch.from_numpy(mask).cuda())
+    value = getattr(ohm, family + "_value")(x, **kw)
+    grads = [[g.cpu().numpy() for g in torch.autograd.grad(value[b], (x, *p), retain_graph=True)]
+             for b in range(len(s))]
+    with torch.no_grad():
+        m = getattr(ohm, family)(x, **kw).cpu().numpy()
+        only = getattr(ohm, family + "_value")(x, **kw).cpu().numpy()
+    value = value.detach().cpu().numpy()
+
+    ref = s.astype(np.float64)
+    top = np.where(mask, -np.inf, ref).max(axis=(1, 2), keepdims=True)
+    ref = np.where(mask, top - (sum(s.shape[1:]) * 80.0 + 200.0) * T, ref)
+    ln = np.tile(np.array(s.shape[1:], np.int32), (len(s), 1))
+    f64 = ORACLE[family](ref, *((go, T) if family == "sw" else (go, ge, T)), ln, prec="f64")
+    assert all(np.isfinite(a).all() for a in (value, only, m, *(g for row in grads for g in row)))
+    assert rel_err(value, f64[0], 1e-3) < 1e-5 and rel_err(only, f64[0], 1e-3) < 1e-5
+    assert abs_err(m, f64[1]) < 1e-4
+    assert abs_err(np.where(mask, 0.0, np.stack([row[0][b] for b, row in enumerate(grads)])), f64[1]) < 1e-4
+    for k in range(len(p) - 1):
+        assert rel_err([float(row[1 + k]) for row in grads], f64[2 + k], 1.0) < 1e-4
