@@ -85,3 +85,27 @@ def test_models_match_the_oracle(family, kind, shape, params, grid, monkeypatch)
     assert abs_err(m, f64[1]) < 1e-4
     for k in range(len(args) - 1):
         assert rel_err(g[:, k], f64[2 + k], 1.0) < 1e-4
+
+
+@pytest.mark.parametrize("grid", ["0", "1"])
+@pytest.mark.parametrize("family", ["sw_affine", *ORACLE])
+def test_blocks_left_out_after_a_failed_attempt(family, grid, monkeypatch):
+    """Long runs of strong matches (attempts fail, the pauses between them grow
+    to 15 blocks) that begin and end inside noise (they shrink again)."""
+    print("attempts", family, "grid", grid, flush=True)
+    monkeypatch.setenv("OHM_GRID", grid)
+    B, L1, L2 = 2, 330, 900
+    rng = np.random.default_rng(12)
+    s = (rng.normal(size=(B, L1, L2)) * 1.5 - 1.0).astype(np.float32)
+    i = np.arange(300)
+    s[0, i, i + 10] += 8.0
+    s[1, i, 2 * i + 200] += 9.0
+    ln = np.tile(np.array([L1, L2], np.int32), (B, 1))
+    go, ge, T = (-1.0, 0.0, 1.0) if family == "sw" else (-11.0, -1.0, 1.0)
+    value, only, m, g = _run(family, s, ln, go, ge, T)
+    args = (go, T) if family == "sw" else (go, ge, T)
+    f64 = {"sw_affine": O.sw_affine_forward, **ORACLE}[family](s.astype(np.float64), *args, ln, prec="f64")
+    assert rel_err(value, f64[0], 1e-3) < 1e-5 and rel_err(only, f64[0], 1e-3) < 1e-5
+    assert abs_err(m, f64[1]) < 1e-4
+    for k in range(len(args) - 1):
+        assert rel_err(g[:, k], f64[2 + k], 1.0) < 1e-4
