@@ -25,8 +25,9 @@ def _kernels(ns: str, soft: str) -> OperatorKernels:
     def prepare(call: KernelCall):
         gap, temp = call.params
         warn_positive_gap(gap, "gap")
-        check_temperature(temp)
-        return (scalar(gap), scalar(temp)), resolve_lengths(call)
+        if call.host is None:
+            check_temperature(temp)
+        return call.host or (scalar(gap), scalar(temp)), resolve_lengths(call)
 
     def forward(call: KernelCall) -> ForwardPass:
         params, lengths = prepare(call)

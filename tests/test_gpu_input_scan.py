@@ -244,3 +244,26 @@ def test_tensor_parameters_read_back_once_check_as_the_torch_path(monkeypatch, g
     torch.cuda.synchronize()
     a, b = outs
     assert (a == b) if isinstance(b, str) else torch.equal(a, b)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("family", ["sw", "sw_affine", "nw", "nw_affine", "sv", "sv_affine"])
+def test_tensor_parameters_are_not_read_again_by_the_adapters(monkeypatch, family):
+    print(f"[gpu case] parameter reads of {family}", flush=True)
+    reads = []
+    host_scalar = _checks.host_scalar
+    monkeypatch.setattr(_checks, "host_scalar", lambda t, name: reads.append(name) or host_scalar(t, name))
+    names = ("gap_open_score", "gap_extend_score") if "affine" in family else ("gap_score",)
+    kw = {n: torch.tensor(-2.0, device=DEV, requires_grad=True) for n in (*names, "temperature")}
+    kw["temperature"] = torch.tensor(1.0, device=DEV, requires_grad=True)
+    x = _scores(7, (3, 20, 24), scale=0.03)
+    value = getattr(ohm, family + "_value")(x, **kw)
+    with torch.no_grad():
+        getattr(ohm, family)(x, **kw)
+        getattr(ohm, family + "_value")(x, **kw)
+    torch.autograd.grad(value.sum(), list(kw.values()))
+    assert reads == []
+    # the map's backward reads what the saved-tensor hooks give back
+    m = getattr(ohm, family)(x, **kw)
+    torch.autograd.grad(m.sum(), [kw["temperature"]])
+    assert len(reads) > 0
