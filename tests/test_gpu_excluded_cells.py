@@ -13,6 +13,7 @@ import torch
 import orihime_amd as ohm
 from helpers import abs_err, rel_err
 from oracle import oracle as O
+from orihime_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -123,3 +124,37 @@ def test_excluded_cells_match_the_oracle(family, kind, shape, monkeypatch):
     assert abs_err(np.where(mask, 0.0, np.stack([row[0][b] for b, row in enumerate(grads)])), f64[1]) < 1e-4
     for k in range(len(p) - 1):
         assert rel_err([float(row[1 + k]) for row in grads], f64[2 + k], 1.0) < 1e-4
+
+
+@pytest.mark.parametrize("grid", ["0", "1"])
+@pytest.mark.parametrize("family", ["sw", "sw_affine"])
+def test_masked_tails_keep_every_pair(family, grid, monkeypatch):
+    """Pairs masked past a last row and column, at every offset from the edges
+    of strips and blocks: none leaves the exponent range (workspace word 8
+    counts the pairs that the log-domain sweeps redo)."""
+    print("masked tails", family, "grid", grid, flush=True)
+    monkeypatch.setenv("OHM_GRID", grid)
+    B, L1, L2 = 64, 200, 150
+    rng = np.random.default_rng(21)
+    s = rng.normal(size=(B, L1, L2)).astype(np.float32)
+    go, ge, t = (-0.75, 0.0, 0.73) if family == "sw" else (-8.0, -0.5, 0.5)
+    ln = np.stack([60 + np.arange(B) * 2, 100 + np.arange(B) % 48], axis=1).astype(np.int32)
+    for b in range(B):
+        s[b, ln[b, 0]:] = s[b, :, ln[b, 1]:] = -(sum(s.shape[1:]) * 80.0 + 200.0) * t
+    x = torch.from_numpy(s).cuda()
+    value, m, g0, g1, g2 = (torch.empty(n, device="cuda") for n in (B, s.shape, B, B, B))
+    ws = torch.empty(_lib.workspace_bytes(family != "sw", _lib.OP_FORWARD, B, L1, L2, -1), dtype=torch.uint8,
+                     device="cuda")
+    if family == "sw":
+        _lib.linear_forward(x, None, None, go, t, value=value, map=m, grad_gap=g0, grad_temp=g2, workspace=ws)
+        f64 = O.sw_forward(s.astype(np.float64), go, t, prec="f64")
+    else:
+        _lib.affine_forward(x, None, None, go, ge, t, value=value, map=m, grad_open=g0, grad_ext=g1, grad_temp=g2,
+                            workspace=ws)
+        f64 = O.sw_affine_forward(s.astype(np.float64), go, ge, t, prec="f64")
+        assert rel_err(g1.cpu().numpy(), f64[3], 1.0) < 1e-4
+    torch.cuda.synchronize()
+    assert int(ws[:256].view(torch.int32)[8].item()) == 0
+    assert rel_err(value.cpu().numpy(), f64[0], 1e-3) < 1e-5
+    assert abs_err(m.cpu().numpy(), f64[1]) < 1e-4
+    assert rel_err(g0.cpu().numpy(), f64[2], 1.0) < 1e-4
