@@ -137,8 +137,14 @@ DEV bool any_greater_i(int a, int b) {
 DEV float ldx(float x, int e) { return __builtin_amdgcn_ldexpf(x, e); }
 DEV int fexp(float x) { return __builtin_amdgcn_frexp_expf(x); }
 // Finite test on the bit pattern (the device code is built without NaN
-// semantics, so isfinite() may be folded away).
-DEV bool finite_bits(float x) { return (__builtin_bit_cast(uint32_t, x) & 0x7f800000u) != 0x7f800000u; }
+// semantics, so isfinite() may be folded away; the empty asm keeps the bits an
+// integer: from the float's own the compiler makes |x| == inf, which a NaN
+// passes as finite).
+DEV bool finite_bits(float x) {
+    uint32_t u = __builtin_bit_cast(uint32_t, x);
+    asm("" : "+v"(u));
+    return (u & 0x7f800000u) != 0x7f800000u;
+}
 
 // Global accesses as (wave-uniform base pointer) + (32-bit lane offset): the
 // compiler emits the scalar-base form, so per-step address updates are scalar
