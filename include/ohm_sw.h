@@ -75,7 +75,9 @@ const char* ohm_version(void);
  * k = 1 after the forward sweep (or tangent forward sweep), k = 2 after the
  * forward sweep's log-domain launch for flagged pairs, k = 3 after the
  * reverse sweep, k = 4 after the reverse sweep's log-domain launch (marks
- * without such a launch are recorded right after the previous one).  NULL
+ * without such a launch are recorded right after the previous one; an affine
+ * forward + reverse call has both log-domain launches between k = 3 and k = 4,
+ * as either sweep may flag a pair).  NULL
  * entries are skipped; count 0 clears the hook (count <= 5).
  * The setting is process-wide and unsynchronised: change it only while no
  * other thread is inside the library, and never while a HIP graph is being

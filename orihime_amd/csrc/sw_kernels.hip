@@ -1696,9 +1696,9 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
     const bool fused = scaled && !grid && need_bwd && use_fused(B, L.a.max_strips);
     const bool team = scaled && !grid && !fused && use_teams(B, L.a.max_strips);
     if (scaled) {
-        // scaled sweep for every pair, then the log-domain sweep for the pairs
-        // it flagged (a launch whose groups only walk the claim list when
-        // none are)
+        // scaled sweeps for every pair, then the log-domain sweeps for the
+        // pairs that either of them flagged (launches that return at once
+        // when none are)
         if (grid) {
             // one fill serves both sweeps (forward entries in words 0..2,
             // reverse entries in words 4..6 of each block)
@@ -1722,6 +1722,21 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
             else OHM_WITH_SH(shared, OHM_DISPATCH_W(L, (sw_affine_scaled_forward_kernel<false, W, kCkpt, SH>)));
         }
         stage_mark(1, L.stream);
+        if (need_bwd) {
+            stage_mark(2, L.stream);
+            if (grid) {
+                OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_groups(sw_affine_scaled_backward_grid<CK, SH>,
+                                                   grid_sweep_lds_bytes(L.a.max_strips), L)));
+                if (st != OHM_OK) return st;
+            } else if (team) {
+                OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_team(sw_affine_scaled_backward_team<CK, SH>,
+                                                   team_sweep_lds_bytes(L.a.max_strips), L)));
+                if (st != OHM_OK) return st;
+            } else if (!fused) {
+                OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, OHM_DISPATCH_W(L, (sw_affine_scaled_backward_kernel<W, CK, SH>))));
+            }
+            stage_mark(3, L.stream);
+        }
         L.a.sel = 1;
         if (need_bwd) OHM_DISPATCH_W(L, (sw_affine_forward_kernel<true, W>));
         else OHM_DISPATCH_W(L, (sw_affine_forward_kernel<false, W>));
@@ -1740,26 +1755,10 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
         else OHM_DISPATCH_W(L, (sw_forward_kernel<false, W>));
     }
     if (!scaled && !lin_scaled) stage_mark(1, L.stream);
-    stage_mark(2, L.stream);
+    if (!scaled || !need_bwd) stage_mark(2, L.stream);
     if ((st = check_launch("forward kernel")) != OHM_OK) return st;
     if (!need_bwd) return OHM_OK;
-    if (scaled) {
-        L.a.sel = 0;
-        if (grid) {
-            OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_groups(sw_affine_scaled_backward_grid<CK, SH>,
-                                               grid_sweep_lds_bytes(L.a.max_strips), L)));
-            if (st != OHM_OK) return st;
-        } else if (team) {
-            OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_team(sw_affine_scaled_backward_team<CK, SH>,
-                                               team_sweep_lds_bytes(L.a.max_strips), L)));
-            if (st != OHM_OK) return st;
-        } else if (!fused) {
-            OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, OHM_DISPATCH_W(L, (sw_affine_scaled_backward_kernel<W, CK, SH>))));
-        }
-        stage_mark(3, L.stream);
-        L.a.sel = 1;
-        OHM_DISPATCH_W(L, (sw_affine_backward_kernel<W>));
-    } else if (affine) {
+    if (affine) {
         OHM_DISPATCH_W(L, (sw_affine_backward_kernel<W>));
     } else if (lin_scaled) {
         stage_mark(3, L.stream);

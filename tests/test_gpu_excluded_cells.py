@@ -158,3 +158,27 @@ def test_masked_tails_keep_every_pair(family, grid, monkeypatch):
     assert rel_err(value.cpu().numpy(), f64[0], 1e-3) < 1e-5
     assert abs_err(m.cpu().numpy(), f64[1]) < 1e-4
     assert rel_err(g0.cpu().numpy(), f64[2], 1.0) < 1e-4
+
+
+@pytest.mark.parametrize("shape", list(SHAPES))
+@pytest.mark.parametrize("rows", [63, 200])
+def test_flagged_pairs_are_redone_in_every_launch_shape(rows, shape, monkeypatch):
+    """Pairs whose scores jump from -75 T to 75 T between adjacent columns leave
+    the exponent range and are redone by the log-domain sweeps, which run after
+    both exponent-tracked ones; the others are not."""
+    print("flagged pairs", rows, shape, flush=True)
+    for k, v in SHAPES[shape].items():
+        monkeypatch.setenv(k, v)
+    rng = np.random.default_rng(rows)
+    s = rng.normal(size=(5, rows, 90)).astype(np.float32)
+    s[1::2] = -75.0
+    s[1::2, :, 40] = 75.0
+    ln = np.tile(np.array([rows, 90], np.int32), (5, 1))
+    ln[2] = [rows - 20, 50]
+    out = [x.cpu().numpy() for x in torch.ops.orihime.soft_sw_affine_with_grads(
+        torch.from_numpy(s).cuda(), -11.0, -1.0, T, torch.from_numpy(ln).cuda())]
+    f64 = O.sw_affine_forward(s.astype(np.float64), -11.0, -1.0, T, ln, prec="f64")
+    assert all(np.isfinite(x).all() for x in out)
+    assert rel_err(out[0], f64[0], 1e-3) < 1e-5
+    assert abs_err(out[1], f64[1]) < 1e-4
+    assert rel_err(out[2], f64[2], 1.0) < 1e-4 and rel_err(out[3], f64[3], 1.0) < 1e-4
