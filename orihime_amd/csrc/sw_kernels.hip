@@ -1601,10 +1601,6 @@ ohm_status launch_groups(K kernel, size_t lds, const Launch& L) {
 // pairs of 512^2 and 512 pairs up to 768^2); teams = 4 / 2 in
 // ohm_set_launch_config or OHM_FUSED=1 / 0 force it on / off.
 bool use_fused(int B, int max_strips) {
-    // its progress words (forward and reverse, 2 x max_strips ints) stay
-    // within the default dynamic LDS of a launch; taller batches run
-    // separate launches (one set of words each)
-    if (2 * (size_t)max_strips * sizeof(int) > 48 * 1024) return false;
     const int cfg = g_cfg_teams.load();
     if (cfg == 4) return true;
     if (cfg != 0) return false;
@@ -1644,9 +1640,7 @@ bool use_ahead(const Launch& L) {
 bool use_model(const SwArgs& a, int model) {
     if (!use_scaled(a)) return false;
     if (model == kSwLinear && env_int("OHM_LINEAR_SCALED", 1) == 0) return false;
-    if (model != kSwLinear && !use_shared(a)) return false;
-    // (the fused launch's progress words)
-    return 2 * (size_t)a.max_strips * sizeof(int) <= 48 * 1024;
+    return model == kSwLinear || use_shared(a);
 }
 template <int MODEL, bool SH>
 ohm_status launch_model(const Launch& L, bool need_bwd) {
@@ -1661,10 +1655,8 @@ ohm_status launch_model(const Launch& L, bool need_bwd) {
         return launch_groups(scaled_backward_grid<MODEL, SH>, lds, L);
     }
     if (need_bwd) {
-        Launch F = L;
-        F.lds = 2 * (size_t)L.a.max_strips * sizeof(int);
-        if (SH && use_ahead(F)) OHM_DISPATCH_W(F, (sw_affine_scaled_fused_ahead_kernel<MODEL, W>));
-        else OHM_DISPATCH_W(F, (scaled_fused_kernel<MODEL, W, SH>));
+        if (SH && use_ahead(L)) OHM_DISPATCH_W(L, (sw_affine_scaled_fused_ahead_kernel<MODEL, W>));
+        else OHM_DISPATCH_W(L, (scaled_fused_kernel<MODEL, W, SH>));
     } else {
         OHM_DISPATCH_W(L, (scaled_value_kernel<MODEL, W, SH>));
     }
@@ -1708,10 +1700,8 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
             else OHM_WITH_SH(shared, st = launch_groups(sw_affine_scaled_forward_grid<false, kCkpt, SH>, lds, L));
             if (st != OHM_OK) return st;
         } else if (fused) {
-            Launch F = L;
-            F.lds = 2 * (size_t)L.a.max_strips * sizeof(int);
-            if (shared && L.ck == kCkpt && use_ahead(F)) OHM_DISPATCH_W(F, (sw_affine_scaled_fused_ahead_kernel<kSwAffine, W>));
-            else OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, OHM_DISPATCH_W(F, (sw_affine_scaled_fused_kernel<W, CK, SH>))));
+            if (shared && L.ck == kCkpt && use_ahead(L)) OHM_DISPATCH_W(L, (sw_affine_scaled_fused_ahead_kernel<kSwAffine, W>));
+            else OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, OHM_DISPATCH_W(L, (sw_affine_scaled_fused_kernel<W, CK, SH>))));
         } else if (team) {
             const size_t lds = team_sweep_lds_bytes(L.a.max_strips);
             if (need_bwd) OHM_WITH_SH(shared, OHM_WITH_CK(L.ck, st = launch_team(sw_affine_scaled_forward_team<true, CK, SH>, lds, L)));

@@ -1,0 +1,48 @@
+"""Batches at the far ends of the sizes a launch takes: pairs of more than
+6144 strips, rows longer than a 32-bit lane offset reaches, border gaps far
+below 2^-2^20.  Against the FP64 oracle, or against the same pair in a smaller
+batch, at the tolerances of the parity tests."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+import orihime_amd as ohm
+from helpers import abs_err, rel_err
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _kernel_names(call):
+    from torch.profiler import ProfilerActivity, profile
+
+    torch.cuda.synchronize()
+    with profile(activities=[ProfilerActivity.CPU, ProfilerActivity.CUDA]) as prof:
+        call()
+        torch.cuda.synchronize()
+    return {getattr(e, "name", "") or getattr(e, "key", "") for e in prof.events()}
+
+
+@pytest.mark.parametrize("grid", ["0", "1"])
+@pytest.mark.parametrize("rows", [64 * 6144 + 1, 983040])
+def test_tall_linear_pairs_run_the_exponent_tracked_sweeps(rows, grid, monkeypatch):
+    print("tall linear pair", rows, "grid", grid, flush=True)
+    monkeypatch.setenv("OHM_GRID", grid)
+    rng = np.random.default_rng(rows)
+    s = rng.normal(size=(1, rows, 3)).astype(np.float32)
+    go, T = -0.75, 0.73
+    x = torch.from_numpy(s).cuda()
+    kw = dict(gap_score=go, temperature=T)
+    out = {}
+
+    def run():
+        out["value"], out["map"] = ohm.sw_value(x, **kw), ohm.sw(x, **kw)
+
+    names = _kernel_names(run)
+    f64 = O.sw_forward(s.astype(np.float64), go, T, prec="f64")
+    assert rel_err(out["value"].cpu().numpy(), f64[0], 1e-3) < 1e-5
+    assert abs_err(out["map"].cpu().numpy(), f64[1]) < 1e-4
+    assert any("scaled" in n for n in names), sorted(n for n in names if "sw" in n)
