@@ -12,6 +12,7 @@ import torch
 import orihime_amd as ohm
 from helpers import abs_err, rel_err
 from oracle import oracle as O
+from orihime_amd import embed
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +47,14 @@ def test_tall_linear_pairs_run_the_exponent_tracked_sweeps(rows, grid, monkeypat
     assert rel_err(out["value"].cpu().numpy(), f64[0], 1e-3) < 1e-5
     assert abs_err(out["map"].cpu().numpy(), f64[1]) < 1e-4
     assert any("scaled" in n for n in names), sorted(n for n in names if "sw" in n)
+
+
+@pytest.mark.parametrize("rows", [64 * 6144 + 1, 740_000, 983040])
+def test_tall_embedding_pairs_fused(rows):
+    print("tall fused embedding pair", rows, flush=True)
+    g = torch.Generator().manual_seed(rows)
+    Q = (torch.randn(1, rows, 32, generator=g) / 32 ** 0.25).to(torch.bfloat16).cuda()
+    K = (torch.randn(1, 3, 32, generator=g) / 32 ** 0.25).to(torch.bfloat16).cuda()
+    ln = torch.tensor([[rows, 3]], dtype=torch.int32).cuda()
+    a, b = (embed.soft_align_embeddings(Q, K, ln, fused=f).cpu().numpy() for f in (True, False))
+    assert np.isfinite(a).all() and rel_err(a, b) < 1e-5
