@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstring>
 #include <string>
@@ -236,12 +237,14 @@ extern "C" ohm_status ohm_scan_inputs(const float* scores, const int32_t* length
     if (B > 0 && cells > 0 && !scores) return fail(OHM_EINVAL, "scores is null");
     hipStream_t s = static_cast<hipStream_t>(stream);
     // in the domain: finite and magnitude <= bound (bits order as magnitudes;
-    // a negative bound admits nothing, a NaN bound every finite cell)
+    // a negative bound admits nothing, -0 the zeros, a NaN bound every finite
+    // cell)
     uint32_t lim = 0x7f800000u;
     if (bound < 0.0f) {
         lim = 0;
     } else if (bound < 3.4028234663852886e38f) {
-        std::memcpy(&lim, &bound, sizeof lim);
+        const float size = std::fabs(bound);  // (-0: its sign bit is no magnitude)
+        std::memcpy(&lim, &size, sizeof lim);
         ++lim;
     }
     if (B <= kSmallPairs && B * cells <= kSmallCells) {

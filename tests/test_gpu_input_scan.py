@@ -247,6 +247,22 @@ def test_tensor_parameters_read_back_once_check_as_the_torch_path(monkeypatch, g
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bound", [0.0, -0.0, -1.0])
+@pytest.mark.parametrize("shape", [(2, 5, 7), (3, 300, 301)])
+def test_scan_with_a_bound_of_zero(shape, bound):
+    print(f"[gpu case] ohm_scan_inputs {shape}, bound {bound!r}", flush=True)
+    x = torch.zeros(shape, device=DEV)
+    x[0, 0, :6] = torch.tensor([1.0, -1.0e4, float("inf"), float("-inf"), float("nan"), -0.0])
+    counts = torch.full((4,), 9, dtype=torch.int32, device=DEV)
+    pmax = torch.full((shape[0],), 9.0, device=DEV)
+    _lib.scan_inputs(x, None, bound, -1.0e4, counts, pmax)
+    torch.cuda.synchronize()
+    # out of the domain: NaN and 1, below zero every finite cell but the marker
+    bad = 2 if bound == 0.0 else x.numel() - 3
+    assert counts.tolist() == [1, bad, 1, 0]
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("family", ["sw", "sw_affine", "nw", "nw_affine", "sv", "sv_affine"])
 def test_tensor_parameters_are_not_read_again_by_the_adapters(monkeypatch, family):
     print(f"[gpu case] parameter reads of {family}", flush=True)
