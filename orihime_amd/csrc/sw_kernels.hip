@@ -1617,6 +1617,10 @@ bool use_scaled(const SwArgs& a) {
     return std::fabs(a.go2) <= 120.0f && std::fabs(a.ge2) <= 120.0f;
 }
 
+// The forward and reverse sweeps also need rows that their 32-bit lane offsets
+// reach; wider batches run the log-domain sweeps.
+bool use_sweeps(const SwArgs& a) { return use_scaled(a) && a.L2max <= kSegmentColumns; }
+
 // Shared-exponent blocks (see sw_affine_scaled.hiph): where a gap opened next
 // to a match and extended over a block stays inside the accepted range
 // (kShLow = 2^-64); beyond it nearly every block would be tried in vain.
@@ -1638,7 +1642,7 @@ bool use_ahead(const Launch& L) {
 // exponent-tracked sweeps (the log-domain ones redo the pairs they flag).
 // The Saigo-Vert and global models have them in shared-exponent form only.
 bool use_model(const SwArgs& a, int model) {
-    if (!use_scaled(a)) return false;
+    if (!use_sweeps(a)) return false;
     if (model == kSwLinear && env_int("OHM_LINEAR_SCALED", 1) == 0) return false;
     return model == kSwLinear || use_shared(a);
 }
@@ -1678,7 +1682,7 @@ ohm_status forward_impl(bool affine, const float* scores, const int32_t* lengths
     L.a.g0 = g0;
     L.a.g1 = g1;
     L.a.g2 = g2;
-    const bool scaled = affine && use_scaled(L.a);
+    const bool scaled = affine && use_sweeps(L.a);
     const bool shared = use_shared(L.a);
     // linear gap: exponent-tracked sweeps, the log-domain sweeps for the pairs
     // they flag; OHM_LINEAR_SCALED=0 keeps the log-domain sweeps alone
@@ -2203,6 +2207,8 @@ extern "C" ohm_status ohm_sw_tangent(const float* scores, const int32_t* lengths
 
 extern "C" ohm_status ohm_embed_offsets(const int32_t* lengths, int32_t B, int32_t Lq, int32_t Lk,
                                         int64_t* offsets, void* stream);
+extern "C" ohm_status ohm_embed_scores(const void* Q, const void* K, const int32_t* lengths, int32_t B, int32_t Lq,
+                                       int32_t Lk, int32_t D, int64_t* offsets, float* scores, void* stream);
 
 extern "C" ohm_status ohm_embed_sw_affine_forward(const void* Q, const void* K, const int32_t* lengths,
                                                   int32_t B, int32_t Lq, int32_t Lk, int32_t D,
@@ -2245,15 +2251,17 @@ extern "C" ohm_status ohm_embed_sw_affine_forward(const void* Q, const void* K, 
         hipLaunchKernelGGL(kernel, dim3(groups), dim3(64 * kW), lds, L.stream, L.a, e);
         return check_launch("embedding sweep kernel");
     };
-    if (D == 32) OHM_WITH_SH(shared, st = launch(embed_sw_fused_kernel<kW, 32, SH>));
+    const bool sweeps = use_sweeps(L.a);
+    if (!sweeps) st = ohm_embed_scores(Q, K, lengths, B, Lq, Lk, D, offsets, scores, stream);
+    else if (D == 32) OHM_WITH_SH(shared, st = launch(embed_sw_fused_kernel<kW, 32, SH>));
     else if (D == 64) OHM_WITH_SH(shared, st = launch(embed_sw_fused_kernel<kW, 64, SH>));
     else OHM_WITH_SH(shared, st = launch(embed_sw_fused_kernel<kW, 128, SH>));
     if (st != OHM_OK) return st;
     stage_mark(1, L.stream);
     stage_mark(2, L.stream);
-    // pairs the scaled sweep flagged: the log-domain sweeps, on the scores
-    // the fused kernel wrote for them
-    L.a.sel = 1;
+    // pairs the scaled sweeps flagged, or all of them: the log-domain sweeps,
+    // on the scores the fused kernel wrote for them
+    L.a.sel = sweeps;
     OHM_DISPATCH_W(L, (sw_affine_forward_kernel<true, W>));
     if ((st = check_launch("embedding fallback forward")) != OHM_OK) return st;
     stage_mark(3, L.stream);

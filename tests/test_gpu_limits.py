@@ -12,7 +12,7 @@ import torch
 import orihime_amd as ohm
 from helpers import abs_err, rel_err
 from oracle import oracle as O
-from orihime_amd import embed
+from orihime_amd import _lib, embed
 
 pytestmark = pytest.mark.gpu
 
@@ -58,3 +58,41 @@ def test_tall_embedding_pairs_fused(rows):
     ln = torch.tensor([[rows, 3]], dtype=torch.int32).cuda()
     a, b = (embed.soft_align_embeddings(Q, K, ln, fused=f).cpu().numpy() for f in (True, False))
     assert np.isfinite(a).all() and rel_err(a, b) < 1e-5
+
+
+# 16 rows of 72 M columns: 60 bytes a column is past 2^32
+WIDE = 72_000_000
+
+
+def test_rows_past_a_32_bit_lane_offset():
+    """The C entry point (the operators bound L1 x L2 further below)."""
+    print("rows of", WIDE, "columns", flush=True)
+    lengths = torch.tensor([[16, 40]], dtype=torch.int32).cuda()
+    small = torch.randn(1, 16, 40, generator=torch.Generator().manual_seed(9)).cuda()
+    x = torch.zeros(1, 16, WIDE, device="cuda")
+    x[:, :, :40] = small
+    go, ge, T = -2.0, -0.5, 0.73
+    value, only, m = torch.empty(1, device="cuda"), torch.empty(1, device="cuda"), torch.empty_like(x)
+    _lib.affine_forward(x, lengths, None, go, ge, T, value=only)
+    _lib.affine_forward(x, lengths, None, go, ge, T, value=value, map=m)
+    f64 = O.sw_affine_forward(small.cpu().numpy().astype(np.float64), go, ge, T, prec="f64")
+    for v in (value, only):
+        assert rel_err(v.cpu().numpy(), f64[0]) < 1e-5
+    assert abs_err(m[:, :, :40].cpu().numpy(), f64[1]) < 1e-4
+    assert not m[:, :, 40:].any()
+    del x, m
+    torch.cuda.empty_cache()
+
+
+def test_fused_embeddings_with_long_key_rows():
+    print("fused embeddings,", WIDE, "keys", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(11)
+    lengths = torch.tensor([[16, 40]], dtype=torch.int32).cuda()
+    Q = torch.randn(1, 16, 32, generator=g, device="cuda").to(torch.bfloat16)
+    K = torch.zeros(1, WIDE, 32, device="cuda", dtype=torch.bfloat16)
+    K[:, :40] = torch.randn(1, 40, 32, generator=g, device="cuda").to(torch.bfloat16)
+    wide = embed.soft_align_embeddings(Q, K, lengths, fused=True)
+    near = embed.soft_align_embeddings(Q, K[:, :40].contiguous(), lengths, fused=True)
+    assert rel_err(wide.cpu().numpy(), near.cpu().numpy()) < 1e-5
+    del K
+    torch.cuda.empty_cache()
