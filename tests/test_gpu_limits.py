@@ -96,3 +96,20 @@ def test_fused_embeddings_with_long_key_rows():
     assert rel_err(wide.cpu().numpy(), near.cpu().numpy()) < 1e-5
     del K
     torch.cuda.empty_cache()
+
+
+@pytest.mark.parametrize("rows", list(range(165_100, 165_301, 20)))
+def test_global_border_gaps_past_the_absent_exponent(rows):
+    """Steep gaps down 165 000 rows, four strong matches: cells, adjoints and
+    the partition near and below 2^-2^20."""
+    print("global pair", rows, "x 4", flush=True)
+    s = np.full((1, rows, 4), -1.0, np.float32)
+    for j in range(4):
+        s[0, (rows // 5) * (j + 1), j] = 60.0
+    kw = dict(gap_open_score=-4.4, gap_extend_score=-4.4, temperature=1.0)
+    x = torch.from_numpy(s).cuda()
+    value, m = ohm.nw_affine_value(x, **kw).cpu().numpy(), ohm.nw_affine(x, **kw).cpu().numpy()
+    f64 = O.nw_affine_forward(s.astype(np.float64), -4.4, -4.4, 1.0, prec="f64")
+    assert rel_err(value, f64[0]) < 1e-5
+    # four matches (the gaps' FP32 sums near 7e5 leave a few percent)
+    assert np.isfinite(m).all() and abs(float(m.sum()) - 4.0) < 0.4
