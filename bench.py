@@ -77,12 +77,12 @@ TRANS_PER_CELL = {"forward": 11, "reverse": 11, "fused": 22}
 BYTES_PER_CELL = {"forward": 4, "reverse": 4, "fused": 8}
 KERNEL_NAMES = {
     "plan": "sw_plan_kernel",
-    "forward": "sw_affine_scaled_forward_kernel<true, W, CK>",
-    "reverse": "sw_affine_scaled_backward_kernel<W, CK>",
+    "forward": "sw_affine_scaled_forward_kernel<true, W, CK, true>",
+    "reverse": "sw_affine_scaled_backward_kernel<W, CK, true>",
     # one launch running each pair's forward and reverse sweep (the launch
     # shape the autotuner picks on the ragged batch); W waves per workgroup,
-    # CK steps between checkpoints
-    "fused": "sw_affine_scaled_fused_kernel<W, CK>",
+    # CK steps between checkpoints, shared-exponent blocks
+    "fused": "sw_affine_scaled_fused_kernel<W, CK, true>",
 }
 
 # The reference's Smith-Waterman shape catalog ("rectangular-production-v1",
@@ -293,23 +293,18 @@ class Launch:
 
 
 def _profiled(name: str, tag: str, kernel: str, shape=None):
-    """Per-launch figure of `kernel` from the `tag:` line of a committed
-    counter profile: the entry of the launch shape (waves, checkpoint stride)
-    when given and present, else the first entry of that kernel."""
+    """Per-launch figure of `kernel` at the launch shape (waves, checkpoint
+    stride) from the `tag:` line of a committed counter profile; None unless
+    the profile holds that very kernel."""
     path = os.path.join(ROOT, "profiles", name)
-    if not os.path.exists(path):
+    if shape is None or not os.path.exists(path):
         return None, None
+    exact = KERNEL_NAMES[kernel].replace("CK", str(shape[1])).replace("W", str(shape[0]))
     for line in open(path):
         if line.startswith(tag + ":"):
             table = json.loads(line.split(":", 1)[1])
-            if shape is not None:
-                exact = KERNEL_NAMES[kernel].replace("CK", str(shape[1])).replace("W", str(shape[0]))
-                if exact in table:
-                    return int(table[exact]), os.path.relpath(path, ROOT)
-            key = KERNEL_NAMES[kernel].split("<")[0] + "<" + ("true" if kernel == "forward" else "")
-            for k, v in table.items():
-                if k.startswith(key):
-                    return int(v), os.path.relpath(path, ROOT)
+            if exact in table:
+                return int(table[exact]), os.path.relpath(path, ROOT)
     return None, None
 
 
