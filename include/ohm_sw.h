@@ -102,8 +102,9 @@ ohm_status ohm_set_launch_config(int32_t waves, int32_t groups_per_cu, int32_t t
  * whole DP tables).  steps: anti-diagonal steps between the checkpoints that
  * the affine forward sweep stores for the reverse sweep (4, 8 or 16; 0 =
  * automatic, 8).  Shorter strides store more and recompute less.  The
- * checkpoints are exact sweep states, so results are bitwise the same for
- * every stride.  The workspace queries use the stride set when they are
+ * checkpoints are exact sweep states, so results do not depend on the stride
+ * (bit for bit where its blocks keep, or all leave, the shared exponent).  The
+ * workspace queries use the stride set when they are
  * called: set it before sizing a workspace.  Process-wide and unsynchronised
  * like ohm_set_launch_config. */
 ohm_status ohm_set_checkpoint_stride(int32_t steps);

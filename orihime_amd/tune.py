@@ -5,11 +5,11 @@ persistent workgroups per CU, per-pair workgroups or wave-scheduled team
 kernels) nor on the tile of the affine sweeps' adjoint (the checkpoint
 stride: anti-diagonal steps per recomputed block, 4, 8 or 16) — only their
 speed does, and the best choice depends on the batch: many mid-size pairs
-favour 4 waves per pair, few long pairs the team or grid kernels; a shorter
+favour 4 waves per pair, few long pairs the grid kernels; a shorter
 stride stores more checkpoints and holds fewer registers per block.
 ``autotune`` times the candidate shapes on the caller's own batch (the best
 of five forward+backward calls each, after a warm-up), then the strides under the
-fastest shape (affine sweeps only: the linear sweeps keep full tables),
+fastest shape (affine sweeps only: the linear sweeps keep 8 steps),
 applies the winner through ``ohm_set_launch_config`` and
 ``ohm_set_checkpoint_stride`` and caches it per batch signature (pair count
 bucket, maximum lengths, layout), so a training loop pays the search once.
